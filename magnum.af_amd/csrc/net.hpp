@@ -19,7 +19,9 @@ struct Net {
     // parameters: per layer W [Cout][Cin][3][3] then b [Cout], concatenated (FP32 masters)
     int64_t nparams{0};
     int64_t woff[kNetLayers]{}, boff[kNetLayers]{};
-    DevBuf master, bf16w, grad, adam_m, adam_v; // bf16w: 16-bit copies of the weights only
+    DevBuf master, packed, grad, adam_m, adam_v;
+    // BF16 weights in MFMA operand order: forward (packoff[0]) and data gradient (packoff[1]) of each layer
+    int64_t packoff[2][kNetLayers]{}, npacked{0};
     DevBuf loss_part, scal;
     double* host_scal{nullptr};
     int64_t adam_t{0};
@@ -36,7 +38,7 @@ struct Net {
     const float* output() const;                  // [B][3][H][W], unit vectors
     double backward(const float* target);         // gradients into grad, returns the loss
     void adam(float lr, float beta1, float beta2, float eps);
-    void sync_bf16();                             // bf16w <- round(master)
+    void sync_bf16();                             // packed <- round(master)
 };
 
 // x [1][8][ny][nx] from m0 (SoA f64, nz = 1) and the five parameter planes; m_out (SoA f64) from
