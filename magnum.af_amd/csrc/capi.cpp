@@ -311,8 +311,9 @@ int mafx_ctx_create(const mafx_mesh* mesh, double Ms, const double* Ms_field_hos
             ctx->py.build(static_cast<int>(ctx->n1));
             ctx->pyh.build(static_cast<int>(mesh->ny)); // the split y transform
             if (ctx->n2 > 1) ctx->pz.build(static_cast<int>(ctx->n2));
-            // the z transform is fused into the tensor product for 2 <= nz <= 8 (nz planes suffice)
-            ctx->nzs = (mesh->nz >= 2 && mesh->nz <= 8) ? mesh->nz : ctx->n2;
+            // the z transform is fused into the tensor product (nz planes suffice) for 2 <= nz <= 8 and,
+            // through LDS columns, for every thickness whose column fits
+            ctx->nzs = (mesh->nz >= 2 && (mesh->nz <= 8 || z_column_fits(ctx.get(), demag_f64(precision)))) ? mesh->nz : ctx->n2;
             const size_t csz = demag_f64(precision) ? sizeof(double2) : sizeof(float2);
             ctx->spec.alloc(csz * 3 * ctx->nzs * ctx->n1 * ctx->hxs);
             MAFX_HIP(hipMemset(ctx->spec.p, 0, ctx->spec.bytes));

@@ -1180,6 +1180,7 @@ void fft_x_forward(mafx_ctx* ctx, const double* in, const double* ms, double sca
         MAFX_HIP(hipGetLastError());
         return;
     }
+    if (mix_x_forward<C>(ctx, in, ms, scale, Xi, Yi, Zi, ncomp, Yr, Zr, out, n2o)) return;
     // Power-of-two rows that fit use the 32 KiB tile under a 6-wave register cap (three resident
     // work-groups per CU), measured faster than the 64 KiB tile at 1024 x 1024 x 4 in both precisions.
     constexpr int E64 = lds_elems<C>();
@@ -1236,6 +1237,7 @@ void fft_x_inverse(mafx_ctx* ctx, const C* spec, int64_t n2s, T* out, double hsc
         MAFX_HIP(hipGetLastError());
         return;
     }
+    if (mix_x_inverse<C, T>(ctx, spec, n2s, out, hscale)) return;
     constexpr int E64 = lds_elems<C>();
     const bool small = is_pow2_plan(desc_of(ph)) && M <= E64 / 2; // as in fft_x_forward
     const int W = lines_per_block(M, small ? E64 / 2 : E64);
@@ -1315,6 +1317,7 @@ void fft_y_split(mafx_ctx* ctx, C* data, int64_t sa, int na, int64_t sb, int nb,
         MAFX_HIP(hipGetLastError());
         return;
     }
+    if (stride == kTile && sa == nb * sb && mix_y_split<C>(ctx, data, na * nb, inv)) return;
     // Tile shapes, measured at 1024 x 1024 x 4 (one column pair = 2 lines): FP32 power-of-two
     // lines of up to E64/2 run 1024-lane work-groups on a 64 KiB tile under an 8-wave register cap
     // (two groups per CU); FP64 ones 1024-lane groups on a 128 KiB tile; both stage the twiddles in

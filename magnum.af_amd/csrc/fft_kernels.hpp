@@ -61,4 +61,19 @@ void tensor_residual_f16(mafx_ctx* ctx, double2* T, const float* Ts, __half2* ou
 void kspace_mul_sym(mafx_ctx* ctx, float2* spec, const float* ts, int64_t n2, const TensorRes* res = nullptr);
 void zfused_sym(mafx_ctx* ctx, float2* spec, const float* ts, int nz, const TensorRes* res = nullptr);
 
+// fft_mixed.hip: the x and y transforms on two-buffer LDS tiles for any length; false where the
+// length has no schedule or a line does not fit, and nothing was launched.  y: nplanes planes [n1][hxs].
+template <class C>
+bool mix_x_forward(mafx_ctx* ctx, const double* in, const double* ms, double scale, int64_t Xi, int64_t Yi, int64_t Zi,
+                   int ncomp, int64_t Yr, int64_t Zr, C* out, int64_t n2o);
+template <class C, class T> bool mix_x_inverse(mafx_ctx* ctx, const C* spec, int64_t n2s, T* out, double hscale);
+template <class C> bool mix_y_split(mafx_ctx* ctx, C* data, int nplanes, bool inv);
+// nz == 1: y forward, tensor product and y inverse in one launch; false where a column does not fit
+bool y_column(mafx_ctx* ctx, double2* spec, const double2* t);
+bool y_column(mafx_ctx* ctx, float2* spec, const float* t, const TensorRes* res);
+// nz > 8: z forward, tensor product and z inverse in one launch, spectrum planes [3][nz]
+bool z_column_fits(const mafx_ctx* ctx, bool f64); // ctx with its mesh and z plan
+void z_column(mafx_ctx* ctx, double2* spec, const double2* t);
+void z_column(mafx_ctx* ctx, float2* spec, const float* t, const TensorRes* res);
+
 } // namespace mafx

@@ -886,8 +886,7 @@ template <class C, class TH, class T> void evaluate_impl(mafx_ctx* ctx, const Ev
         const double* ms = (!ctx->atom_dipole && ctx->has_ms_field) ? ctx->ms_field.as<double>() : nullptr;
         const double scale = ctx->atom_dipole ? 1.0 : (ctx->has_ms_field ? 1.0 : ctx->Ms);
         fft_x_forward<C>(ctx, a.m, ms, scale, g.nx, g.ny, g.nz, 3, g.ny, g.nz, spec, nzs);
-        // column tiles: rows ky are kTile elements apart, planes n1 hxs
-        fft_y_split<C>(ctx, spec, sa, 3, n1 * hxs, static_cast<int>(g.nz), kTile, false);
+        // y transforms: column tiles, rows ky are kTile elements apart, planes n1 hxs
         // tensor product: complex reference spectrum (FP64) or its real symmetric quarter (FP32)
         // (plus, MAFX_TERM_FULL_TENSOR, the FP16 residual that makes it the reference's spectrum)
         TensorRes res{};
@@ -897,14 +896,29 @@ template <class C, class TH, class T> void evaluate_impl(mafx_ctx* ctx, const Ev
             for (int c = 0; c < 6; ++c) res.inv[c] = ctx->res_inv[c];
             resp = &res;
         }
+        auto y_pass = [&](bool inv) { fft_y_split<C>(ctx, spec, sa, 3, n1 * hxs, static_cast<int>(g.nz), kTile, inv); };
         auto kmul = [&](int64_t planes) {
             if constexpr (std::is_same<C, float2>::value)
                 kspace_mul_sym(ctx, spec, ctx->tensor.as<float>(), planes, resp);
             else
                 kspace_mul<C>(ctx, spec, ctx->tensor.as<C>(), sa);
         };
+        bool column = false; // a single layer's y stage as one pass
         if (n2 == 1) {
+            if constexpr (std::is_same<C, float2>::value)
+                column = y_column(ctx, spec, ctx->tensor.as<float>(), resp);
+            else
+                column = y_column(ctx, spec, ctx->tensor.as<C>());
+        }
+        if (!column) y_pass(false);
+        if (column) {
+        } else if (n2 == 1) {
             kmul(1);
+        } else if (nzs == g.nz && g.nz > 8) {
+            if constexpr (std::is_same<C, float2>::value)
+                z_column(ctx, spec, ctx->tensor.as<float>(), resp);
+            else
+                z_column(ctx, spec, ctx->tensor.as<C>());
         } else if (nzs == g.nz) {
             if constexpr (std::is_same<C, float2>::value)
                 zfused_sym(ctx, spec, ctx->tensor.as<float>(), static_cast<int>(g.nz), resp);
@@ -917,7 +931,7 @@ template <class C, class TH, class T> void evaluate_impl(mafx_ctx* ctx, const Ev
             fft_strided<C>(ctx, ctx->pz, spec, sa, 3, kTile, static_cast<int>(n1), n1 * hxs, static_cast<int>(n2),
                            static_cast<int>(g.nz), true, sizeof(C) == 8 ? "fft_z_inv_f32" : "fft_z_inv_f64");
         }
-        fft_y_split<C>(ctx, spec, sa, 3, n1 * hxs, static_cast<int>(g.nz), kTile, true);
+        if (!column) y_pass(true);
         const double P_total = static_cast<double>(ctx->n0) * n1 * n2;
         const double hscale = (ctx->atom_dipole ? ctx->Ms : 1.0) / P_total;
         TH* hd = ctx->hdem.as<TH>();
