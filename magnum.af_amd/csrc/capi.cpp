@@ -319,10 +319,11 @@ int mafx_ctx_create(const mafx_mesh* mesh, double Ms, const double* Ms_field_hos
             MAFX_HIP(hipMemset(ctx->spec.p, 0, ctx->spec.bytes));
             ctx->hdem.alloc((demag_f64(precision) ? sizeof(double) : sizeof(float)) * 3 * N);
             build_tensor(ctx.get());
+            slab_prepare(ctx.get());
         }
         ctx->device_bytes = static_cast<int64_t>(ctx->ms_field.bytes + ctx->partials.bytes + ctx->scal.bytes +
                                                  ctx->hbuf.bytes + ctx->spec.bytes + ctx->tensor.bytes +
-                                                 ctx->hdem.bytes);
+                                                 ctx->hdem.bytes + ctx->slab_part.bytes + ctx->slab_count.bytes);
         for (auto& t : ctx->terms)
             ctx->device_bytes += static_cast<int64_t>(term_bytes(t));
         *out = ctx.release();

@@ -75,5 +75,10 @@ bool y_column(mafx_ctx* ctx, float2* spec, const float* t, const TensorRes* res)
 bool z_column_fits(const mafx_ctx* ctx, bool f64); // ctx with its mesh and z plan
 void z_column(mafx_ctx* ctx, double2* spec, const double2* t);
 void z_column(mafx_ctx* ctx, float2* spec, const float* t, const TensorRes* res);
+// fft_slab.hip: y and z stages of films of a few layers in one launch.  slab_prepare stores the built
+// tensor as that kernel's rows and sets ctx->slab where the mesh has one; slab_column runs it.
+void slab_prepare(mafx_ctx* ctx);
+void slab_column(mafx_ctx* ctx, double2* spec);
+void slab_column(mafx_ctx* ctx, float2* spec);
 
 } // namespace mafx

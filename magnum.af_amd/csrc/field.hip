@@ -944,8 +944,10 @@ template <class C, class TH, class T> void evaluate_impl(mafx_ctx* ctx, const Ev
             else
                 kspace_mul<C>(ctx, spec, ctx->tensor.as<C>(), sa);
         };
-        bool column = false; // a single layer's y stage as one pass
-        if (n2 == 1) {
+        bool column = ctx->slab; // the stages between the x transforms as one pass
+        if (column) {
+            slab_column(ctx, spec);
+        } else if (n2 == 1) {
             if constexpr (std::is_same<C, float2>::value)
                 column = y_column(ctx, spec, ctx->tensor.as<float>(), resp);
             else

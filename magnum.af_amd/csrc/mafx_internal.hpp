@@ -173,6 +173,9 @@ struct mafx_ctx {
     // FP32 path: [6][n2h] planes of n1h hxs real f32, the mirror-symmetric spectrum (fft.hip).
     // Planes store columns in tiles of 4 (tcol, fft_device.hpp).
     mafx::DevBuf tensor;
+    bool slab{false};         // the tensor is stored as the rows of fft_slab.hip, which runs the y and z stages
+    int slab_split{0};        // its columns shared by several groups, their partial sums and counters
+    mafx::DevBuf slab_part, slab_count;
     int64_t res_off{0};       // MAFX_TERM_FULL_TENSOR: byte offset of the FP16 residual in `tensor`
     float res_inv[6]{};       // ... and its per-component 1 / scale
     mafx::DevBuf spec;        // [3][nzs] planes of n1 hxs complex values, column tiles
