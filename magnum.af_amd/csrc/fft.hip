@@ -386,7 +386,11 @@ __global__ void __launch_bounds__(BS, MINW)
     C* buf = reinterpret_cast<C*>(smem_raw);
     C* tws = buf + lds_padded(E);
     for (int t = threadIdx.x; t < M / 2; t += BS) tws[t] = twh[t]; // half table: w^(t + M/2) = -w^t
-    const uint32_t grp = blockIdx.x, zc = fdiv(grp, gyd), yg = grp - zc * gyd.d;
+    // a group whose rows fill only part of the 128-byte lines of a column tile (2048-point rows) shares
+    // them with its neighbour: both behind one L2 (FP32 2048 x 1024 x 8: 220 -> 176 us)
+    constexpr bool PART = W * kTile * sizeof(C) < 128;
+    const uint32_t grp = PART ? xcd_swizzle(blockIdx.x, gridDim.x) : blockIdx.x;
+    const uint32_t zc = fdiv(grp, gyd), yg = grp - zc * gyd.d;
     const uint32_t c = fdiv(zc, nzd), z = zc - c * nzd.d;
     const int y0 = static_cast<int>(yg) << LOGW;
     const C* srow = spec + (static_cast<int64_t>(c) * n2s + z) * plane + kTile * y0;
