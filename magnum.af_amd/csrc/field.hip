@@ -42,6 +42,8 @@ struct EpiTerm {
     const double* aex;
     const uint32_t* ridx;
     const void* rkw; // 6N RKKY weights per neighbour in the stencils' type T, or null
+    const uint8_t* rki; // or N indices into ..
+    const void* rkt;    // .. the table [256][8] of the cells' distinct six weights
     const double* pf; // N: D_constants (DMI) or Ku1_field (UNIAXIAL), or null
     const double* ax; // 3N: normalised Ku1_axis_field (UNIAXIAL), or null
 };
@@ -50,7 +52,7 @@ struct EpiParams {
     int64_t nx, ny, nz, N;
     const double* m;
     const double* ms; // Ms_field or null
-    double Ms;
+    double Ms, Ms_inv;
     double ex_w[3], ex_self; // exchange filter (exchange_field.cpp:116-125)
     double dmi_c[3];         // 1 / (2 d) central difference weights (dmi_field.cpp:53-64)
     double rk_pref[3];       // mu0 * d^2 of the RKKY couplings: dx^2 for x AND y, dz^2 for z
@@ -94,6 +96,17 @@ template <class U> __device__ __forceinline__ void stb(U* base, uint32_t boff, U
 template <class T> struct V3 {
     T x, y, z;
 };
+
+// The kernel's parameters (its first argument), read again where they are used: what a z step needs would
+// otherwise be loaded before the loop, and the 100 to 250 scalars that do not fit the registers are kept
+// in lanes of vector registers, at one vector instruction per use (the RKKY list at 2048 x 1024 x 8: 110
+// -> 78 registers, and with the weights as table indices and one reciprocal of Ms 314 -> 260 us).
+__device__ __forceinline__ const EpiParams& params_here() {
+    using K = const __attribute__((address_space(4))) EpiParams*;
+    K p = (K)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const EpiParams*)p;
+}
 
 // Sum over the block of `nv` per-thread values with a fixed tree, written to partials[s][blk].
 __device__ void block_reduce_store(double* vals, int nv, const int* is_max, double* partials, int64_t nblocks) {
@@ -354,14 +367,20 @@ __device__ __forceinline__ void cell_terms(const EpiParams& P, int64_t x, int64_
             bool pre = false;
             // the neighbour weights precomputed once per term (k_rkky_weights), summed in the
             // order of the in-kernel form below (an absent neighbour's weight is 0)
-            if (tm.rkw) {
+            if (tm.rki || tm.rkw) {
                 pre = true;
-                const T* wp = static_cast<const T*>(tm.rkw);
-                const uint32_t ot = static_cast<uint32_t>(i) * static_cast<uint32_t>(sizeof(T));
                 constexpr int ord[6] = {1, 0, 3, 2, 5, 4};
                 T w[6];
+                if (tm.rki) {
+                    const T* wp = static_cast<const T*>(tm.rkt) + 8 * tm.rki[i];
 #pragma unroll
-                for (int k = 0; k < 6; ++k) w[k] = ldb(wp + ord[k] * N, ot);
+                    for (int k = 0; k < 6; ++k) w[k] = wp[ord[k]];
+                } else {
+                    const T* wp = static_cast<const T*>(tm.rkw);
+                    const uint32_t ot = static_cast<uint32_t>(i) * static_cast<uint32_t>(sizeof(T));
+#pragma unroll
+                    for (int k = 0; k < 6; ++k) w[k] = ldb(wp + ord[k] * N, ot);
+                }
 #pragma unroll
                 for (int k = 0; k < 6; ++k) {
                     const double wk = static_cast<double>(w[k]);
@@ -407,9 +426,16 @@ __device__ __forceinline__ void cell_terms(const EpiParams& P, int64_t x, int64_
                 zc(z > 0, i - sxy, 4);
             }
             if (!P.ms) {
-                h0 = static_cast<T>(a0 / P.Ms);
-                h1 = static_cast<T>(a1 / P.Ms);
-                h2 = static_cast<T>(a2 / P.Ms);
+                if constexpr (sizeof(T) == 4) {
+                    // one FP64 reciprocal from the host: its last bit is far below the rounding to FP32
+                    h0 = static_cast<T>(a0 * P.Ms_inv);
+                    h1 = static_cast<T>(a1 * P.Ms_inv);
+                    h2 = static_cast<T>(a2 * P.Ms_inv);
+                } else {
+                    h0 = static_cast<T>(a0 / P.Ms);
+                    h1 = static_cast<T>(a1 / P.Ms);
+                    h2 = static_cast<T>(a2 / P.Ms);
+                }
             } else if (msi != 0) {
                 h0 = static_cast<T>(a0 / msi);
                 h1 = static_cast<T>(a1 / msi);
@@ -602,7 +628,7 @@ __global__ void __launch_bounds__(kBlock, MINW) k_epi_cells(EpiParams P, FastDiv
 // group's cells at the same z (one halo cell each side, loaded by the edge lanes), so only the
 // centre, the next z and the two y neighbours are read from memory, 9 loads per cell instead
 // of 21.  Zero padding as in cell_epilogue.
-template <class T, class TH, bool RED, uint64_t PROG, int MINW>
+template <class T, class TH, bool RED, uint64_t PROG, int MINW, bool HERE = RED>
 __global__ void __launch_bounds__(kBlock, MINW) k_epi_zcol(EpiParams P, FastDiv bprd) {
     __shared__ V3<T> row[kBlock + 2];
     const int nx = static_cast<int>(P.nx), ny = static_cast<int>(P.ny), nz = static_cast<int>(P.nz);
@@ -648,7 +674,7 @@ __global__ void __launch_bounds__(kBlock, MINW) k_epi_zcol(EpiParams P, FastDiv 
         __syncthreads();
         if (valid) {
             const V3<T> nb[6] = {row[t], (x + 1 < nx) ? row[t + 2] : V3<T>{0, 0, 0}, to_t(ym), to_t(yp), prev, to_t(nxt)};
-            cell_terms<T, RED, PROG>(P, x, y, z, cur[0], cur[1], cur[2], nb, hd, acc);
+            cell_terms<T, RED, PROG>(HERE ? params_here() : P, x, y, z, cur[0], cur[1], cur[2], nb, hd, acc);
         }
         prev = to_t(cur);
 #pragma unroll
@@ -737,7 +763,7 @@ __global__ void __launch_bounds__(kBlock, MINW) k_epi_col4(EpiParams P, FastDiv 
             const V3<T> nb[6] = {tile[z][ty + 1][tx], tile[z][ty + 1][tx + 2], tile[z][ty][tx + 1], tile[z][ty + 2][tx + 1],
                                  z > 0 ? tile[z > 0 ? z - 1 : 0][ty + 1][tx + 1] : zero,
                                  z + 1 < nz ? tile[z + 1 < kColZ ? z + 1 : z][ty + 1][tx + 1] : zero};
-            cell_terms<T, false, PROG>(P, x, y, z, c[z][0], c[z][1], c[z][2], nb, hd[z], acc);
+            cell_terms<T, false, PROG>(params_here(), x, y, z, c[z][0], c[z][1], c[z][2], nb, hd[z], acc);
         }
     }
 }
@@ -800,12 +826,99 @@ __global__ void __launch_bounds__(256) k_rkky_weights(const double* __restrict__
     for (int k = 0; k < 6; ++k) w[k * N + i] = static_cast<W>(wk[k]);
 }
 
+// A multilayer has few distinct materials, so most meshes have few distinct sets of six weights: each cell
+// then stores the place of its set in a hash table of 256 (keys: a 64-bit hash of the set, 0 = free)
+// instead of the set.  flag: more sets than places, or two of one hash.
+template <class W> __device__ __forceinline__ uint64_t rkky_hash(const W (&v)[6]) {
+    uint64_t h = 0x9E3779B97F4A7C15ull;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        uint64_t b;
+        if constexpr (sizeof(W) == 4)
+            b = __float_as_uint(v[k]);
+        else
+            b = static_cast<uint64_t>(__double_as_longlong(v[k]));
+        h = (h ^ b) * 0xFF51AFD7ED558CCDull;
+        h ^= h >> 32;
+    }
+    return h ? h : 1;
+}
+constexpr int kRkkySets = 256;
+template <class W>
+__global__ void __launch_bounds__(256) k_rkky_sets(const W* __restrict__ w, int64_t N, unsigned long long* keys,
+                                                   W* __restrict__ table, uint8_t* __restrict__ index, int* flag) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= N || __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return;
+    W v[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) v[k] = w[k * N + i];
+    const unsigned long long h = rkky_hash(v);
+    int s = static_cast<int>(h & (kRkkySets - 1));
+    for (int probe = 0; probe < 64; ++probe, s = (s + 1) & (kRkkySets - 1)) {
+        unsigned long long have = __hip_atomic_load(keys + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (have == 0) {
+            have = atomicCAS(keys + s, 0ull, h);
+            if (have == 0)
+                for (int k = 0; k < 6; ++k) table[8 * s + k] = v[k];
+        }
+        if (have == 0 || have == h) {
+            index[i] = static_cast<uint8_t>(s);
+            return;
+        }
+    }
+    __hip_atomic_store(flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// every cell's set against the table's, bit for bit
+template <class W>
+__global__ void __launch_bounds__(256) k_rkky_check(const W* __restrict__ w, int64_t N, const W* __restrict__ table,
+                                                    const uint8_t* __restrict__ index, int* flag) {
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (i >= N) return;
+    using B = typename std::conditional<sizeof(W) == 4, uint32_t, uint64_t>::type;
+    const B* a = reinterpret_cast<const B*>(w) + i;
+    const B* b = reinterpret_cast<const B*>(table) + 8 * index[i];
+    bool same = true;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) same = same && a[k * N] == b[k];
+    if (!same) *flag = 1;
+}
+// Replaces t.rkw by the indexed form where the sets fit: 1 instead of 24 bytes read per cell in FP32 (48
+// in FP64); the weights are the same to the last bit.
+template <class W> void rkky_index(mafx_ctx* ctx, TermDev& t) {
+    const int64_t N = ctx->N;
+    DevBuf keys, flag;
+    keys.alloc(sizeof(unsigned long long) * kRkkySets);
+    flag.alloc(sizeof(int));
+    t.rkt.alloc(sizeof(W) * 8 * kRkkySets);
+    t.rki.alloc(static_cast<size_t>(N));
+    MAFX_HIP(hipMemsetAsync(keys.p, 0, keys.bytes, ctx->stream));
+    MAFX_HIP(hipMemsetAsync(flag.p, 0, flag.bytes, ctx->stream));
+    MAFX_HIP(hipMemsetAsync(t.rki.p, 0, t.rki.bytes, ctx->stream));
+    MAFX_HIP(hipMemsetAsync(t.rkt.p, 0, t.rkt.bytes, ctx->stream));
+    hipLaunchKernelGGL(k_rkky_sets<W>, dim3(grid_for(N, 256)), dim3(256), 0, ctx->stream, t.rkw.as<W>(), N,
+                       keys.as<unsigned long long>(), t.rkt.as<W>(), t.rki.as<uint8_t>(), flag.as<int>());
+    hipLaunchKernelGGL(k_rkky_check<W>, dim3(grid_for(N, 256)), dim3(256), 0, ctx->stream, t.rkw.as<W>(), N, t.rkt.as<W>(),
+                       t.rki.as<uint8_t>(), flag.as<int>());
+    MAFX_HIP(hipGetLastError());
+    int over = 0;
+    MAFX_HIP(hipMemcpyAsync(&over, flag.p, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+    MAFX_HIP(hipStreamSynchronize(ctx->stream));
+    if (over) {
+        t.rki.release();
+        t.rkt.release();
+    } else {
+        t.rkw.release();
+    }
+}
+
 } // namespace
 
 void rkky_weights(mafx_ctx* ctx, TermDev& t) {
     const mafx_mesh& g = ctx->mesh;
     const int64_t N = ctx->N;
     const bool f32 = stencils_f32(ctx->precision);
+    t.rki.release();
+    t.rkt.release();
     t.rkw.alloc((f32 ? sizeof(float) : sizeof(double)) * 6 * N);
     // the same prefactors as make_params: mu0 dx^2 couples x AND y neighbours, mu0 dz^2 the layers
     const double pxy = kMu0 * std::pow(g.dx, 2), pz = kMu0 * std::pow(g.dz, 2);
@@ -819,7 +932,10 @@ void rkky_weights(mafx_ctx* ctx, TermDev& t) {
                            t.rkky.as<double>(), t.aex.as<double>(), ridx, g.nx, g.ny, g.nz, pxy, pxy, pz,
                            t.rkw.as<double>());
     MAFX_HIP(hipGetLastError());
-    MAFX_HIP(hipStreamSynchronize(ctx->stream));
+    if (f32)
+        rkky_index<float>(ctx, t);
+    else
+        rkky_index<double>(ctx, t);
 }
 
 namespace {
@@ -834,6 +950,7 @@ EpiParams make_params(mafx_ctx* ctx, const EvalArgs& a, int64_t nblocks) {
     P.m = a.m;
     P.ms = ctx->has_ms_field ? ctx->ms_field.as<double>() : nullptr;
     P.Ms = ctx->Ms;
+    P.Ms_inv = 1.0 / ctx->Ms;
     P.ex_w[0] = 1 / std::pow(g.dx, 2);
     P.ex_w[1] = 1 / std::pow(g.dy, 2);
     P.ex_w[2] = 1 / std::pow(g.dz, 2);
@@ -860,6 +977,8 @@ EpiParams make_params(mafx_ctx* ctx, const EvalArgs& a, int64_t nblocks) {
         e.aex = td.aex.as<double>();
         e.ridx = td.has_ridx ? td.ridx.as<uint32_t>() : nullptr;
         e.rkw = td.rkw.p;
+        e.rki = td.rki.as<uint8_t>();
+        e.rkt = td.rkt.p;
         e.pf = td.pfield.p ? td.pfield.as<double>() : nullptr;
         e.ax = td.axfield.p ? td.axfield.as<double>() : nullptr;
         if (e.pf || e.ax) P.has_fields = 1;
@@ -1062,11 +1181,16 @@ template <class C, class TH, class T> void evaluate_impl(mafx_ctx* ctx, const Ev
                     ctx->scal_nterms = P.nterms;
                     return;
                 }
-                KZ kz = k_epi_zcol<T, TH, false, 0, MWW>;
-                if (prog == kP1) kz = k_epi_zcol<T, TH, false, kP1, MWZ>;
-                if (prog == kP2) kz = k_epi_zcol<T, TH, false, kP2, MWZ>;
-                if (prog == kP3) kz = k_epi_zcol<T, TH, false, kP3, MWW>;
-                if (prog == kP4) kz = k_epi_zcol<T, TH, false, kP4, MWZ>;
+                // LLG stages read their parameters ahead of the loop (with params_here 111 -> 118 us at 1024 x 1024 x 4)
+                const auto pick = [&](auto here) -> KZ {
+                    constexpr bool HERE = decltype(here)::value;
+                    return prog == kP1   ? k_epi_zcol<T, TH, false, kP1, MWZ, HERE>
+                           : prog == kP2 ? k_epi_zcol<T, TH, false, kP2, MWZ, HERE>
+                           : prog == kP3 ? k_epi_zcol<T, TH, false, kP3, MWW, HERE>
+                           : prog == kP4 ? k_epi_zcol<T, TH, false, kP4, MWZ, HERE>
+                                         : k_epi_zcol<T, TH, false, 0, MWW, HERE>;
+                };
+                const KZ kz = P.mode == static_cast<int>(OutMode::LLG) ? pick(std::false_type{}) : pick(std::true_type{});
                 const int64_t ng = g.ny * bpr;
                 hipLaunchKernelGGL(kz, dim3(static_cast<unsigned>(ng)), dim3(kBlock), 0, ctx->stream, P,
                                    make_fastdiv(static_cast<uint32_t>(bpr)));
