@@ -296,8 +296,7 @@ int mafx_ctx_create(const mafx_mesh* mesh, double Ms, const double* Ms_field_hos
         // memory order), vector reductions
         int64_t nblk = std::max<int64_t>(mesh->ny * mesh->nz * ((mesh->nx + 255) / 256), (N + 255) / 256);
         nblk = std::max<int64_t>(nblk, reduction_partials_needed(3 * N));
-        ctx->partials.alloc(sizeof(double) * 10 * nblk);
-        ctx->scal.alloc(sizeof(double) * 64);
+        ctx->partials.alloc(sizeof(double) * (10 * nblk + reduction_partials_extra()));
         MAFX_HIP(hipHostMalloc(reinterpret_cast<void**>(&ctx->host_scal), sizeof(double) * 64, hipHostMallocDefault));
         ctx->hbuf.alloc(sizeof(double) * 3 * N);
         if (ctx->demag_term >= 0) {
@@ -321,7 +320,7 @@ int mafx_ctx_create(const mafx_mesh* mesh, double Ms, const double* Ms_field_hos
             build_tensor(ctx.get());
             slab_prepare(ctx.get());
         }
-        ctx->device_bytes = static_cast<int64_t>(ctx->ms_field.bytes + ctx->partials.bytes + ctx->scal.bytes +
+        ctx->device_bytes = static_cast<int64_t>(ctx->ms_field.bytes + ctx->partials.bytes +
                                                  ctx->hbuf.bytes + ctx->spec.bytes + ctx->tensor.bytes +
                                                  ctx->hdem.bytes + ctx->slab_part.bytes + ctx->slab_count.bytes);
         for (auto& t : ctx->terms)

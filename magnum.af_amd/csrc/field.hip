@@ -768,28 +768,6 @@ __global__ void __launch_bounds__(kBlock, MINW) k_epi_col4(EpiParams P, FastDiv 
     }
 }
 
-// Fixed-order reduction of partials[s][0..nb) into out[s].
-__global__ void k_reduce_slots(const double* __restrict__ partials, int64_t nb, int nslots, int nsum,
-                               double* __restrict__ out) {
-    __shared__ double red[kBlock];
-    const int s = blockIdx.x;
-    if (s >= nslots) return;
-    const bool is_max = s >= nsum;
-    double v = is_max ? 0.0 : 0.0;
-    for (int64_t b = threadIdx.x; b < nb; b += kBlock) {
-        const double p = partials[s * nb + b];
-        v = is_max ? fmax(v, p) : v + p;
-    }
-    red[threadIdx.x] = v;
-    __syncthreads();
-    for (int w = kBlock / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] = is_max ? fmax(red[threadIdx.x], red[threadIdx.x + w])
-                                                       : red[threadIdx.x] + red[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[s] = red[0];
-}
-
 template <class C> C* spec_of(mafx_ctx* ctx) { return ctx->spec.as<C>(); }
 
 // RKKY stencil weights of cell i towards its six neighbours (x-, x+, y-, y+, z-, z+; 0 where the
@@ -1249,18 +1227,14 @@ void evaluate(mafx_ctx* ctx, const EvalArgs& a) {
 
 // Reduces the partials of the last evaluate() (energy slots and, in gradient mode, the two
 // maxima) to host values.  E_terms is indexed by the context's term order.
-int finish_energy_launch(mafx_ctx* ctx) {
+int finish_energy_launch(mafx_ctx* ctx, const double* g, const double* d, int64_t n) {
     const int nt = ctx->scal_nterms;
-    const int nslots = nt + 2;
-    hipLaunchKernelGGL(k_reduce_slots, dim3(nslots), dim3(kBlock), 0, ctx->stream, ctx->partials.as<double>(),
-                       ctx->scal_nblocks, nslots, nt, ctx->scal.as<double>());
-    MAFX_HIP(hipGetLastError());
-    return nslots;
+    reduce_slots(ctx, ctx->scal_nblocks, nt + 2, nt, g, d, n);
+    return nt + 2;
 }
 
 void finish_energy(mafx_ctx* ctx, uint32_t mask, double* E_terms, double* E_total) {
-    const int nslots = finish_energy_launch(ctx);
-    MAFX_HIP(hipMemcpyAsync(ctx->host_scal, ctx->scal.p, sizeof(double) * nslots, hipMemcpyDeviceToHost, ctx->stream));
+    finish_energy_launch(ctx);
     MAFX_HIP(hipStreamSynchronize(ctx->stream));
     finish_energy_combine(ctx, mask, E_terms, E_total);
 }

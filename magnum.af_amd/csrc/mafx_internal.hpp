@@ -183,7 +183,6 @@ struct mafx_ctx {
     mafx::DevBuf hdem;        // [3][N] FFT-convolution field (f64 or f32) between the x inverse and the cell pass
     mafx::DevBuf hbuf;        // 3N f64 scratch (field output for helpers)
     mafx::DevBuf partials;    // reduction partials (f64)
-    mafx::DevBuf scal;        // small device scalars
     // LBFGS two-loop step whose final reduction (its dot product, alpha_i and coefficient) is
     // still pending in partials: the next two-loop pass forms it, or lbfgs_flush launches it
     struct LbfgsPending {
@@ -195,7 +194,8 @@ struct mafx_ctx {
         double* coef{nullptr};
         double* dot{nullptr};
     } lbfgs_pend;
-    double* host_scal{nullptr}; // pinned host scalars (hipHostMalloc)
+    double* host_scal{nullptr}; // pinned host scalars (hipHostMalloc), written by the reductions' last kernels
+    mafx::DevBuf lbfgs_work;    // the LBFGS vectors of the last run, kept while they are small (lbfgs.cpp)
     int64_t scal_nblocks{0};  // partial-sum blocks of the last evaluation
     int scal_nterms{0};       // terms selected in the last evaluation
     double last_max_torque{0}, last_max_h{0}; // max|m x H|, max|H| of the last gradient evaluation
@@ -254,9 +254,10 @@ struct EvalArgs {
 // are reduced by finish_energy.
 void evaluate(mafx_ctx* ctx, const EvalArgs& a);
 void finish_energy(mafx_ctx* ctx, uint32_t mask, double* E_terms, double* E_total);
-// The two halves of finish_energy: the reduction into ctx->scal[0, slots) (returns the slot count),
-// and the term energies from those slots once they are in ctx->host_scal.
-int finish_energy_launch(mafx_ctx* ctx);
+// The two halves of finish_energy: the reduction into ctx->host_scal[0, slots) (returns the slot count;
+// with g also g . d and max |g| over n elements, into the two slots behind them), and the term energies
+// from those slots once the stream has been synchronised.
+int finish_energy_launch(mafx_ctx* ctx, const double* g = nullptr, const double* d = nullptr, int64_t n = 0);
 void finish_energy_combine(mafx_ctx* ctx, uint32_t mask, double* E_terms, double* E_total);
 void build_tensor(mafx_ctx* ctx);
 

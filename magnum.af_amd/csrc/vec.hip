@@ -94,6 +94,37 @@ __global__ void __launch_bounds__(kB) k_final(const double* __restrict__ part, i
     if (threadIdx.x == 0) out[s] = v;
 }
 
+// Fixed-order reduction of partials[s][0..nb) into out[s], sums for s < nsum, else maxima; the groups
+// from nslots on reduce the sum and the maximum of k_dot_maxabs' partials as k_final does.
+__global__ void __launch_bounds__(kB) k_reduce_slots(const double* __restrict__ partials, int64_t nb, int nslots, int nsum,
+                                                     const double* __restrict__ part2, int nb2, double* __restrict__ out) {
+    const int s = blockIdx.x;
+    if (s >= nslots) {
+        const bool mx = s > nslots;
+        const double* p = part2 + (s - nslots) * nb2;
+        double v = 0;
+        for (int i = threadIdx.x; i < nb2; i += kB) v = mx ? fmax(v, p[i]) : v + p[i];
+        v = mx ? block_max(v) : block_sum(v);
+        if (threadIdx.x == 0) out[s] = v;
+        return;
+    }
+    __shared__ double red[kB];
+    const bool is_max = s >= nsum;
+    double v = 0.0;
+    for (int64_t b = threadIdx.x; b < nb; b += kB) {
+        const double p = partials[s * nb + b];
+        v = is_max ? fmax(v, p) : v + p;
+    }
+    red[threadIdx.x] = v;
+    __syncthreads();
+    for (int w = kB / 2; w > 0; w >>= 1) {
+        if (threadIdx.x < w) red[threadIdx.x] = is_max ? fmax(red[threadIdx.x], red[threadIdx.x + w])
+                                                       : red[threadIdx.x] + red[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) out[s] = red[0];
+}
+
 // util.cpp:34 (a / |a|) and util.cpp:37-42 (zero vectors stay zero)
 __global__ void __launch_bounds__(kB) k_normalize(double* __restrict__ m, int64_t N, int zero_safe) {
     const int64_t i = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x;
@@ -327,8 +358,9 @@ __global__ void __launch_bounds__(kB) k_sub(double* __restrict__ out, const doub
     if (i < n) out[i] = a[i] - b[i];
 }
 
-double read_scalar(mafx_ctx* ctx, int nslots) {
-    MAFX_HIP(hipMemcpyAsync(ctx->host_scal, ctx->scal.p, sizeof(double) * nslots, hipMemcpyDeviceToHost, ctx->stream));
+// The reductions' last kernels write to pinned host memory: a copy would be another launch, about 5 us
+// of each step and line search.
+double read_scalar(mafx_ctx* ctx) {
     MAFX_HIP(hipStreamSynchronize(ctx->stream));
     return ctx->host_scal[0];
 }
@@ -342,10 +374,10 @@ double dot(mafx_ctx* ctx, const double* a, const double* b, int64_t n) {
         ProfScope ps(ctx, "dot_f64", 16.0 * n);
         hipLaunchKernelGGL(k_dot, dim3(nb), dim3(kB), 0, ctx->stream, a, b, n, ctx->partials.as<double>());
         hipLaunchKernelGGL(k_final, dim3(1), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(),
-                           static_cast<int>(nb), 1, 1, ctx->scal.as<double>());
+                           static_cast<int>(nb), 1, 1, ctx->host_scal);
     }
     MAFX_HIP(hipGetLastError());
-    return read_scalar(ctx, 1);
+    return read_scalar(ctx);
 }
 
 double max_abs(mafx_ctx* ctx, const double* a, int64_t n) {
@@ -355,10 +387,10 @@ double max_abs(mafx_ctx* ctx, const double* a, int64_t n) {
         ProfScope ps(ctx, "maxabs_f64", 8.0 * n);
         hipLaunchKernelGGL(k_maxabs, dim3(nb), dim3(kB), 0, ctx->stream, a, n, ctx->partials.as<double>());
         hipLaunchKernelGGL(k_final, dim3(1), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(),
-                           static_cast<int>(nb), 1, 0, ctx->scal.as<double>());
+                           static_cast<int>(nb), 1, 0, ctx->host_scal);
     }
     MAFX_HIP(hipGetLastError());
-    return read_scalar(ctx, 1);
+    return read_scalar(ctx);
 }
 
 void normalize(mafx_ctx* ctx, double* m, bool zero_safe) {
@@ -372,9 +404,9 @@ void mean_m(mafx_ctx* ctx, const double* m, double out[3]) {
     const unsigned nb = red_blocks(ctx->N);
     hipLaunchKernelGGL(k_mean, dim3(nb), dim3(kB), 0, ctx->stream, m, ctx->N, ctx->partials.as<double>());
     hipLaunchKernelGGL(k_final, dim3(4), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(), static_cast<int>(nb), 4,
-                       4, ctx->scal.as<double>());
+                       4, ctx->host_scal);
     MAFX_HIP(hipGetLastError());
-    read_scalar(ctx, 4);
+    read_scalar(ctx);
     for (int c = 0; c < 3; ++c) out[c] = ctx->host_scal[c] / ctx->host_scal[3];
 }
 
@@ -443,13 +475,17 @@ void dot_dev(mafx_ctx* ctx, const double* a, const double* b, int64_t n, double*
     MAFX_HIP(hipGetLastError());
 }
 
-void dot_max_dev(mafx_ctx* ctx, const double* a, const double* b, int64_t n, double* out_dev) {
+void reduce_slots(mafx_ctx* ctx, int64_t nblocks, int nslots, int nsum, const double* a, const double* b, int64_t n) {
     lbfgs_flush(ctx);
     const unsigned nb = red_blocks(n);
-    ProfScope ps(ctx, "dot_max_f64", 16.0 * n);
-    hipLaunchKernelGGL(k_dot_maxabs, dim3(nb), dim3(kB), 0, ctx->stream, a, b, n, ctx->partials.as<double>());
-    hipLaunchKernelGGL(k_final, dim3(2), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(), static_cast<int>(nb),
-                       2, 1, out_dev);
+    // behind the evaluation's partials, which are not reduced yet
+    double* part2 = ctx->partials.as<double>() + ctx->partials.bytes / sizeof(double) - 2 * kMaxRedBlocks;
+    if (a) {
+        ProfScope ps(ctx, "dot_max_f64", 16.0 * n);
+        hipLaunchKernelGGL(k_dot_maxabs, dim3(nb), dim3(kB), 0, ctx->stream, a, b, n, part2);
+    }
+    hipLaunchKernelGGL(k_reduce_slots, dim3(nslots + (a ? 2 : 0)), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(),
+                       nblocks, nslots, nsum, part2, static_cast<int>(nb), ctx->host_scal);
     MAFX_HIP(hipGetLastError());
 }
 void max_abs_dev(mafx_ctx* ctx, const double* a, int64_t n, double* out_dev) {
@@ -671,13 +707,6 @@ void axpy_dev(mafx_ctx* ctx, double* y, const double* a_dev, const double* x, in
     MAFX_HIP(hipGetLastError());
 }
 
-void read_device(mafx_ctx* ctx, const double* src_dev, int n, double* dst_host) {
-    lbfgs_flush(ctx);
-    MAFX_HIP(hipMemcpyAsync(ctx->host_scal, src_dev, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-    MAFX_HIP(hipStreamSynchronize(ctx->stream));
-    for (int i = 0; i < n; ++i) dst_host[i] = ctx->host_scal[i];
-}
-
 void llg_rhs(mafx_ctx* ctx, double alpha, double dt, const double* m, const double* h, double* k) {
     hipLaunchKernelGGL(k_llg_rhs, dim3(grid_for(ctx->N, kB)), dim3(kB), 0, ctx->stream, m, h, k, ctx->N, alpha, dt);
     MAFX_HIP(hipGetLastError());
@@ -794,10 +823,10 @@ double rk_error(mafx_ctx* ctx, const double* m, const void* const* k, const doub
         else
             rk_error_k<double, 1>(ctx, m, a, ns, rkf_form, sumbk, len, nb);
         hipLaunchKernelGGL(k_final, dim3(1), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(),
-                           static_cast<int>(nb), 1, 0, ctx->scal.as<double>());
+                           static_cast<int>(nb), 1, 0, ctx->host_scal);
     }
     MAFX_HIP(hipGetLastError());
-    return read_scalar(ctx, 1);
+    return read_scalar(ctx);
 }
 
 void accept(mafx_ctx* ctx, double* m, const double* dm, bool normalize_m, bool zero_safe) {
@@ -825,5 +854,6 @@ void copy(mafx_ctx* ctx, double* dst, const double* src, int64_t n) {
 
 // the widest reductions over n entries use 5 slots (lbfgs_pair)
 int64_t reduction_partials_needed(int64_t n) { return static_cast<int64_t>(red_blocks(n)) * 5; }
+int64_t reduction_partials_extra() { return 2 * kMaxRedBlocks; }
 
 } // namespace mafx

@@ -18,19 +18,19 @@ void scale(mafx_ctx* ctx, double* y, double a, int64_t n);
 void sub(mafx_ctx* ctx, double* out, const double* a, const double* b, int64_t n);
 void copy(mafx_ctx* ctx, double* dst, const double* src, int64_t n);
 int64_t reduction_partials_needed(int64_t n);
+int64_t reduction_partials_extra(); // doubles at the end of the partials, beside an evaluation's own
 // Device-side scalars (no host synchronisation): *out_dev = a . b and max |a| with the kernels and
-// reduction tree of dot() / max_abs(), y += (*a_dev) x, and one read of n device doubles.
+// reduction tree of dot() / max_abs(), y += (*a_dev) x.
 void dot_dev(mafx_ctx* ctx, const double* a, const double* b, int64_t n, double* out_dev);
 void max_abs_dev(mafx_ctx* ctx, const double* a, int64_t n, double* out_dev);
-// out_dev[0] = a . b and out_dev[1] = max |a| in one pass over a, each bit for bit as dot_dev /
-// max_abs_dev form it
-void dot_max_dev(mafx_ctx* ctx, const double* a, const double* b, int64_t n, double* out_dev);
+// The evaluation's slots [0, nslots) to ctx->host_scal (sums for s < nsum, then maxima) and, with a,
+// a . b and max |a| to the two slots behind them, each bit for bit as dot_dev / max_abs_dev form it.
+void reduce_slots(mafx_ctx* ctx, int64_t nblocks, int nslots, int nsum, const double* a, const double* b, int64_t n);
 void axpy_dev(mafx_ctx* ctx, double* y, const double* a_dev, const double* x, int64_t n);
-void read_device(mafx_ctx* ctx, const double* src_dev, int n, double* dst_host);
 // LBFGS fused vector work, bit for bit the unfused sequence's results:
 // lbfgs_fused: q_out = (q_in + (*coef_dev) v) [* scale] (negated when `negate`), *out_dev = dnext . q
 //   (before negation), with dot()'s tree; coef_dev null skips the axpy.  q_out may alias q_in.
-// lbfgs_pair: s = m - x_old, y = g - g_old, out_dev[0..4] = y.s, y.y, s.s, max|s|, max|m|.
+// lbfgs_pair: s = m - x_old, y = g - g_old, out[0..4] (device or pinned host memory) = y.s, y.y, s.s, max|s|, max|m|.
 // neg_copy: y = -x.
 // mode 1 / 2 also forms the next step's scalars from the dot product d = *out_dev, as lbfgs_alpha
 // (alpha_i = rho d, coef = -alpha_i) / lbfgs_beta (coef = alpha_i - rho d) would, in the same launch
@@ -45,7 +45,7 @@ void lbfgs_fused(mafx_ctx* ctx, const double* q_in, const double* coef_dev, cons
 void lbfgs_dot_alpha(mafx_ctx* ctx, const double* a, const double* b, int64_t n, double* dot_out, double rho,
                      double* alpha_i, double* coef);
 void lbfgs_pair(mafx_ctx* ctx, const double* m, const double* x_old, const double* g, const double* g_old,
-                double* s, double* y, int64_t n, double* out_dev);
+                double* s, double* y, int64_t n, double* out);
 void neg_copy(mafx_ctx* ctx, double* y, const double* x, int64_t n);
 // <m> of mafx_mean_m with its partial sums in a static device array: no allocation, no
 // synchronisation, result in out_dev[0..2] (device memory), launched on `stream`.
