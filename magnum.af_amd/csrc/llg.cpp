@@ -237,9 +237,9 @@ double attempt(mafx_llg* L, const double* m, double t, double dt, const char* sc
     // per-cell pass that produces k_(s-1) (the stage combination of adaptive_runge_kutta.cpp:
     // 138-164 with k_(s-1) still in registers, so no pass re-reads it); the inputs alternate
     // between two buffers, since a pass still reads its own input's neighbours.  Results are the
-    // separate pass's to the last bit.  DP78, and meshes below 2^20 cells (where the per-cell
-    // pass has too few lanes to hide the extra loads: 256 x 128 x 4 runs 8% slower fused), form
-    // them in a pass of their own.
+    // separate pass's to the last bit.  DP78, and meshes whose per-cell pass
+    // has too few lanes to hide the extra loads (mafx_ctx::rk_fuse_min_cells), form them in a pass of
+    // their own.
     const bool fused = T.stages <= kMaxRkFused + 1 && ctx->N >= ctx->rk_fuse_min_cells;
     double* stage_in[2] = {L->mtmp.as<double>(), L->mtmp2.as<double>()};
     auto next_input = [&](int s) { // s: the stage whose input the pass being set up writes

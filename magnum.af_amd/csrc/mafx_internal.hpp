@@ -153,8 +153,10 @@ struct mafx_ctx {
     mafx::DevBuf ms_field; // N f64
     int precision{MAFX_F64};
     int num_cus{256};         // compute units of the current device (persistent grids)
-    // RK stage inputs are formed in the per-cell pass from this many cells on (below it the
-    // pass has too few lanes to hide the extra loads); MAFX_RK_FUSE_MIN_CELLS overrides it
+    // RK stage inputs are formed in the per-cell pass from this many cells on where that pass walks z
+    // columns of several layers (below it has too few lanes to hide the extra loads: 512 x 32 x 4 297
+    // against 318 us a step), and always where it has a lane per cell (1024 x 256 x 1 350 -> 329,
+    // 100 x 25 x 1 210 -> 203); MAFX_RK_FUSE_MIN_CELLS overrides it
     int64_t rk_fuse_min_cells{int64_t{1} << 20};
     // MAFX_F32_FIELD integrators keep their stage derivatives k_j in FP32 (MAFX_RK_K64=1: FP64)
     bool rk_k32{true};
@@ -250,6 +252,8 @@ struct EvalArgs {
     int rk_n{0};
     double* rk_out{nullptr};
 };
+// Whether the per-cell pass of fields and LLG stages walks z columns of several layers (field.hip).
+bool cells_on_z_columns(const mafx_ctx* ctx);
 // Runs the selected terms on m; the energy partial sums (one per term) land in ctx->partials and
 // are reduced by finish_energy.
 void evaluate(mafx_ctx* ctx, const EvalArgs& a);
