@@ -1145,6 +1145,15 @@ void allow_lds(const void* fn, size_t bytes) {
 
 } // namespace
 
+// Power-of-two rows below the compile-time shapes: the in-place kernels where their tiles of up to 64 rows
+// give half of the CUs a group, else the per-mesh tiles of fft_mixed.hip (the same sums).  FP64, us, per-mesh
+// -> in-place: 128 x 300 x 4 forward 15.1 -> 10.5, inverse 11.6 -> 7.9; 64 x 512 x 3 12.3 -> 9.8, 7.6 -> 6.8.
+template <class C> bool inplace_rows(const mafx_ctx* ctx, const FftPlan& ph, int64_t rows) {
+    constexpr int E = lds_elems<C>();
+    if (!is_pow2_plan(desc_of(ph)) || ph.L > E / 2) return false;
+    return rows / lines_per_block(ph.L, E / 2) >= ctx->num_cus / 2;
+}
+
 template <class C>
 void fft_x_forward(mafx_ctx* ctx, const double* in, const double* ms, double scale, int64_t Xi, int64_t Yi,
                    int64_t Zi, int ncomp, int64_t Yr, int64_t Zr, C* out, int64_t n2o) {
@@ -1184,13 +1193,13 @@ void fft_x_forward(mafx_ctx* ctx, const double* in, const double* ms, double sca
         MAFX_HIP(hipGetLastError());
         return;
     }
-    if (mix_x_forward<C>(ctx, in, ms, scale, Xi, Yi, Zi, ncomp, Yr, Zr, out, n2o)) return;
+    const int64_t rows = static_cast<int64_t>(ncomp) * Zr * Yr;
+    if (!inplace_rows<C>(ctx, ph, rows) && mix_x_forward<C>(ctx, in, ms, scale, Xi, Yi, Zi, ncomp, Yr, Zr, out, n2o)) return;
     // Power-of-two rows that fit use the 32 KiB tile under a 6-wave register cap (three resident
     // work-groups per CU), measured faster than the 64 KiB tile at 1024 x 1024 x 4 in both precisions.
     constexpr int E64 = lds_elems<C>();
     const bool small = is_pow2_plan(desc_of(ph)) && M <= E64 / 2;
     const int W = lines_per_block(M, small ? E64 / 2 : E64);
-    const int64_t rows = static_cast<int64_t>(ncomp) * Zr * Yr;
     require(rows * (M + 1) < (int64_t{1} << 31) && Xi < (int64_t{1} << 30), "x transform: too many rows");
     const unsigned grid = static_cast<unsigned>((rows + W - 1) / W);
     const double bytes = static_cast<double>(rows) * (Xi * 8.0 + ctx->hx * sizeof(C));
@@ -1241,11 +1250,11 @@ void fft_x_inverse(mafx_ctx* ctx, const C* spec, int64_t n2s, T* out, double hsc
         MAFX_HIP(hipGetLastError());
         return;
     }
-    if (mix_x_inverse<C, T>(ctx, spec, n2s, out, hscale)) return;
+    const int64_t rows = 3 * g.nz * g.ny;
+    if (!inplace_rows<C>(ctx, ph, rows) && mix_x_inverse<C, T>(ctx, spec, n2s, out, hscale)) return;
     constexpr int E64 = lds_elems<C>();
     const bool small = is_pow2_plan(desc_of(ph)) && M <= E64 / 2; // as in fft_x_forward
     const int W = lines_per_block(M, small ? E64 / 2 : E64);
-    const int64_t rows = 3 * g.nz * g.ny;
     require(rows * (M + 1) < (int64_t{1} << 31), "x transform: too many rows");
     const unsigned grid = static_cast<unsigned>((rows + W - 1) / W);
     const double bytes = static_cast<double>(rows) * (ctx->hx * sizeof(C) + g.nx * sizeof(T));

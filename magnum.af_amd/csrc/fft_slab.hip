@@ -35,6 +35,7 @@ namespace mafx {
 
 namespace {
 
+constexpr int kSlabShared = 2; // columns of a last round that several groups share, at most
 constexpr int kSlabPad = 16; // tensor entries between classes 0 (k <= Q / 2) and S / 2
 
 template <class C, int NZ, int LOGN, int LOGS> struct SlabShape {
@@ -423,10 +424,15 @@ template <class C, int NZ, int LOGN> SlabPlan<C> slab_plan_of() {
 //   FP32 512 x 64 x 4 44 -> 26, 1024 x 256 x 2 67 -> 49, 512 x 512 x 4 100 -> 90, 1024 x 1024 x 4 353 -> 302;
 //   FP64 512 x 128 x 2 55 -> 36, 512 x 512 x 4 249 -> 218, 1024 x 1024 x 4 1050 -> 883.
 // Left out: FP32 1024 x 1024 x 8 742 -> 915, 100 x 512 x 8 71 -> 77, FP64 512 x 512 x 8 500 -> 632,
-// 100 x 1024 x 4 132 -> 159.
+// 100 x 1024 x 4 132 -> 159, 64 x 512 x 3 50 -> 51; and, where a group has a CU to itself, meshes whose
+// last round of columns is nearly empty (260 x 1024 x 2 FP32 76 -> 90, 260 x 256 x 3 FP64 73 -> 83).
 template <class C> SlabPlan<C> slab_plan(int nx, int ny, int nz, int cus) {
     constexpr bool F64 = sizeof(C) == sizeof(double2);
-    if (nx < cus && (ny == 1024 ? F64 || nz == 4 : ny == 512 && nz == 8)) return {};
+    const int hx = nx + 1, rounds = (hx + cus - 1) / cus;
+    const bool heavy = ny == 1024 || (ny == 512 && nz == 8) || (F64 && ny == 256 && nz > 2);
+    if (nx < cus && (ny == 1024 ? F64 || nz == 4 || 3 * nx < cus : ny == 512 && (nz == 8 || (F64 && nz > 2 && 3 * nx < cus))))
+        return {};
+    if (heavy && rounds > 1 && hx % cus > kSlabShared && 4 * hx < 3 * rounds * cus) return {};
     switch (100 * ny + nz) {
 #define MAFX_SLAB(NZ, LOGN) \
     case 100 * (1 << LOGN) + NZ: return slab_plan_of<C, NZ, LOGN>();
@@ -492,7 +498,7 @@ template <class C> void slab_rows(mafx_ctx* ctx) {
     // (1024 x 1024 x 4: 308 -> 302 us in FP32, 937 -> 874 in FP64.  Each sharing group writes its L2 back:
     // with all 101 columns of 100 x 512 x 4 shared the field takes 139 us instead of 44.)
     const int tail = static_cast<int>(ctx->hx % ctx->num_cus);
-    ctx->slab_split = ctx->hx > ctx->num_cus && tail <= 2 ? tail : 0;
+    ctx->slab_split = ctx->hx > ctx->num_cus && tail <= kSlabShared ? tail : 0;
     if (ctx->slab_split > 0) {
         ctx->slab_part.alloc(sizeof(C) * ctx->slab_split * p.S * (p.S / 2 * 8) * p.block);
         ctx->slab_count.alloc(sizeof(int) * ctx->slab_split);
