@@ -21,7 +21,7 @@
 // lanes, one for the even and one for the odd kz, which halves the registers it needs; their inverses are
 // added across the pair.
 //
-// At 1024 x 1024 x 4 FP32 the pass takes 183 us (the three it replaces 219) and moves 370 MB, 74 us at
+// At 1024 x 1024 x 4 FP32 the pass takes 183 us (the three it replaces 219) and moves 357 MB, 71 us at
 // the copy rate; vector instructions take 80 us and LDS 70 us, and one group of 12 waves per CU overlaps
 // them little.  80 registers and two groups per CU (the column read again per class) spill and take twice
 // as long.  FP64: 699 us against 850, bound by the tensor's bytes (320 us) and the latency of its loads.
