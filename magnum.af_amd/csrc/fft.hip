@@ -1135,7 +1135,7 @@ void allow_lds(const void* fn, size_t bytes) {
     static std::mutex mu;
     static std::map<const void*, size_t> granted;
     if (bytes <= 65536) return;
-    require(bytes <= 160 * 1024, "kernel LDS request exceeds 160 KiB");
+    require(bytes <= kLdsMax, "kernel LDS request exceeds 160 KiB");
     std::lock_guard<std::mutex> lk(mu);
     size_t& g = granted[fn];
     if (g >= bytes) return;
@@ -1299,7 +1299,6 @@ void fft_y_split(mafx_ctx* ctx, C* data, int64_t sa, int na, int64_t sb, int nb,
     const FftDesc d = desc_of(ph);
     constexpr int E64 = lds_elems<C>();
     constexpr bool kF32 = sizeof(C) == sizeof(float2);
-    constexpr size_t kLdsMax = 160 * 1024;
     // compile-time shapes: power-of-two M of 256..1024 on 8192-element tiles of whole column tiles
     // (1024 lanes; FP32 under an 8-wave register cap, two groups per CU; FP64 one group per CU)
     if (stride == kTile && ctx->n1 == 2 * M && (M == 256 || M == 512 || M == 1024)) {

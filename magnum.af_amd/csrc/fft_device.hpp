@@ -14,6 +14,7 @@
 #include <hip/hip_runtime.h>
 
 #include "fastdiv.hpp"
+#include "mix_tiles.hpp"
 
 namespace mafx {
 
@@ -52,8 +53,6 @@ __host__ __device__ inline int64_t tcol(int64_t kx, int64_t n1T) { return (kx >>
 // groups of W lanes at a stride of R W elements, a multiple of the bank count for the power-of-two
 // shapes here; the padding spreads consecutive groups over different banks.
 __device__ __forceinline__ int lds_pad(int i) { return i + (i >> 5); }
-// LDS elements to allocate for n logical elements
-constexpr int lds_padded(int n) { return n + (n >> 5) + 1; }
 
 // R-point DFT in registers; forward uses w = exp(-2 pi i / R), inverse its conjugate.
 // Generic odd radices read w_R^p = tw[p L / R] from the length-L table.

@@ -26,8 +26,6 @@ namespace mafx {
 
 namespace {
 
-constexpr size_t kLdsMax = 160 * 1024;
-
 // The schedule with the fewest stages and, among those, the smallest largest radix.  Powers of two
 // keep the radix-8 schedule of FftPlan, whose results the compile-time shaped kernels share.
 void mix_plan(int L, std::vector<int>& best) {
@@ -87,14 +85,7 @@ bool reproducible(const mafx_ctx* ctx, int L) { return !ctx->atom_dipole || (L &
 // Whether the schedule covers the length (a length of 1 needs no stage).
 bool scheduled(const MixDesc& d) { return d.L == 1 || d.nstages > 0; }
 
-// LDS of a tile of `lines` lines: two buffers, the stage twiddles w_L^t and, unless the kernel has
-// no second table, the packing or split twiddles w_2L^t, t <= L
-template <class C> size_t mix_lds(int L, int lines, bool second = true) {
-    return (2 * static_cast<size_t>(lds_padded(L * lines)) + L + (second ? L + 1 : 0)) * sizeof(C);
-}
-
-// Lanes for a tile of n elements: one per eight, in whole waves, at most 512
-int mix_block(int64_t n) { return static_cast<int>(std::min<int64_t>(512, std::max<int64_t>(64, (n / 8 + 63) / 64 * 64))); }
+template <class C> size_t mix_lds(int L, int lines, bool second = true) { return mix_lds_bytes(sizeof(C), L, lines, second); }
 
 // Groups a launch should have before its tiles may grow: three per CU
 int64_t mix_fill(const mafx_ctx* ctx) { return 3 * static_cast<int64_t>(ctx->num_cus); }
@@ -313,8 +304,7 @@ __device__ __forceinline__ void tensor_product(const TensorArg<C>& a, int kx, in
 // y < ny.  One launch and one pass over half the spectrum instead of three over all of it.  The even
 // and the odd ky (the split of k_mix_y_fwd) are transformed together (NH = 2) or, where six lines per
 // column do not fit a useful tile, one after the other (NH = 1): the first half's outputs then wait
-// in registers, at most ACC per lane.
-constexpr int kColAcc = 8;
+// in registers, at most kColAcc per lane (col_tile).
 template <class C, int FORM, int NH>
 __global__ void __launch_bounds__(512)
     k_col(C* __restrict__ spec, int64_t plane, TensorArg<C> ta, int hx, FastDiv Wd, FastDiv lined, MixDesc d, FastDiv Md,
@@ -658,30 +648,17 @@ template <class C, int FORM> bool col_launch(mafx_ctx* ctx, C* spec, const Tenso
     const MixDesc& d = mix_desc(ctx->pyh.L);
     const int M = d.L, hx = static_cast<int>(ctx->hx);
     if (!scheduled(d)) return false;
-    // both halves at once while two groups fit a CU; W: columns per group
-    const auto lines = [](int nh, int w) { return 3 * nh * w; };
-    int W = 0, NH = 2;
-    for (int nh : {2, 1}) {
-        for (int w : {4, 2, 1}) {
-            const bool fits = mix_lds<C>(M, lines(nh, w)) <= (nh == 1 && w == 1 ? kLdsMax : size_t{56} * 1024) &&
-                              (nh == 2 || 3 * M * w <= kColAcc * 512);
-            if (fits && (w == 1 || (hx + w - 1) / w >= mix_fill(ctx))) {
-                W = w;
-                NH = nh;
-                break;
-            }
-        }
-        if (W) break;
-    }
+    const ColTile t = col_tile(sizeof(C), M, hx, mix_fill(ctx));
+    const int W = t.W, NH = t.NH, lines = 3 * NH * W;
     if (W == 0) return false;
+    require(NH == 2 || 3 * M * W <= kColAcc * t.block, "y column: more outputs than its lanes keep");
     ProfScope ps(ctx, nm("ycol_mul_f32", "ycol_mul_f64", sizeof(C)),
                  6.0 * static_cast<double>(M) * ctx->hx * sizeof(C) + tensor_bytes<C>(ctx, FORM == kFull, FORM == kSymRes));
-    const size_t lds = mix_lds<C>(M, lines(NH, W));
+    const size_t lds = mix_lds<C>(M, lines);
     auto fn = NH == 2 ? k_col<C, FORM, 2> : k_col<C, FORM, 1>;
     allow_lds(reinterpret_cast<const void*>(fn), lds);
-    const int bs = NH == 2 ? mix_block(M * lines(NH, W)) : std::max(mix_block(M * lines(NH, W)), (3 * M * W / kColAcc + 63) / 64 * 64);
-    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>((hx + W - 1) / W)), dim3(bs), lds, ctx->stream, spec,
-                       ctx->nzs * ctx->n1 * ctx->hxs, ta, hx, make_fastdiv(W), make_fastdiv(lines(NH, W)), d,
+    hipLaunchKernelGGL(fn, dim3(static_cast<unsigned>((hx + W - 1) / W)), dim3(t.block), lds, ctx->stream, spec,
+                       ctx->nzs * ctx->n1 * ctx->hxs, ta, hx, make_fastdiv(W), make_fastdiv(lines), d,
                        make_fastdiv(M), tw_of<C>(ctx->pyh), tw_of<C>(ctx->py));
     MAFX_HIP(hipGetLastError());
     return true;
