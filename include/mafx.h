@@ -160,7 +160,8 @@ int mafx_ctx_destroy(mafx_ctx* ctx);
 /* Launch on an existing HIP stream (hipStream_t passed as void*); NULL selects the null stream. */
 int mafx_ctx_set_stream(mafx_ctx* ctx, void* stream);
 int mafx_ctx_sync(mafx_ctx* ctx);
-/* Device bytes held by the context (tensor, FFT workspace, parameters). */
+/* Device bytes held by the context (tensor, FFT workspace, parameters and, after an LBFGS run, the work
+ * space kept for the next one, at most 256 MiB). */
 int mafx_ctx_device_bytes(const mafx_ctx* ctx, int64_t* bytes);
 /* Time of the State the next field and energy evaluations see (State::t, state.hpp), used by
  * time-dependent ExternalField callbacks only.  The integrator sets it per RK stage itself. */

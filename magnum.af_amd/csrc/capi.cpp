@@ -351,7 +351,7 @@ int mafx_ctx_sync(mafx_ctx* ctx) {
 }
 
 int mafx_ctx_device_bytes(const mafx_ctx* ctx, int64_t* bytes) {
-    return guarded([&] { *bytes = ctx->device_bytes; });
+    return guarded([&] { *bytes = ctx->device_bytes + static_cast<int64_t>(ctx->lbfgs_work.bytes); });
 }
 
 int mafx_ctx_set_time(mafx_ctx* ctx, double t) {
