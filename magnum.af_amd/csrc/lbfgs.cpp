@@ -299,12 +299,15 @@ int lbfgs_minimize(mafx_ctx* ctx, double* m, double tolerance, int64_t max_iter,
     const size_t vec_bytes = (bytes + 255) / 256 * 256, work_bytes = kVectors * vec_bytes + 16 * sizeof(double);
     struct Work {
         mafx_ctx* ctx;
-        DevBuf buf; // the context's while the run lasts
+        mafx_ctx* moved{nullptr}; // the finish context, once the run is on it
+        DevBuf buf;               // the context's while the run lasts
         explicit Work(mafx_ctx* c, size_t b) : ctx(c), buf(std::move(c->lbfgs_work)) {
             if (buf.bytes < b) buf.alloc(b);
         }
         ~Work() {
-            (void)hipStreamSynchronize(ctx->stream); // also where an exception ends the run
+            // no work on the vectors is left queued, also where an exception ends the run
+            (void)hipStreamSynchronize(ctx->stream);
+            if (moved) (void)hipStreamSynchronize(moved->stream);
             if (buf.bytes <= kKeep) ctx->lbfgs_work = std::move(buf);
         }
     } work(ctx, work_bytes);
@@ -510,6 +513,7 @@ int lbfgs_minimize(mafx_ctx* ctx, double* m, double tolerance, int64_t max_iter,
             // gradient replace the stalled context's, and the next iteration starts from them
             move_now = false;
             MAFX_HIP(hipStreamSynchronize(ctx->stream));
+            work.moved = finish_ctx;
             ctx = finish_ctx;
             L.ctx = finish_ctx;
             f = L.energy_and_gradient(mcur, gcur);
