@@ -68,6 +68,27 @@ def test_shared_columns(n, cus, precision, monkeypatch):
 
 
 @pytest.mark.parametrize("precision", ["f64", "f32"])
+def test_shared_columns_on_a_side_stream(precision, monkeypatch):
+    """A context created and used at once on a stream of its own, which does not wait for the null stream."""
+    import torch
+    print(f"\n[shared columns, side stream] {precision}", flush=True)
+    monkeypatch.setenv("MAFX_NUM_CUS", "3")
+    M = mf()
+    n = (4, 512, 4)
+    g = M.Mesh(*n, 2e-9, 2.5e-9, 3e-9)
+    state = M.State(g, 1.1e6, rand_m(n, 35))
+    term = M.DemagField(g)
+    ref = state._context([term], precision).heff(state.m_dev).cpu().numpy()
+    side = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        ctx = M.Context(g, 1.1e6, None, [term], precision)
+        h = ctx.heff(state.m_dev)
+        side.synchronize()
+        assert np.array_equal(h.cpu().numpy().view(np.uint64), ref.view(np.uint64))
+
+
+@pytest.mark.parametrize("precision", ["f64", "f32"])
 @pytest.mark.parametrize("n", [(256, 256, 5), (64, 1024, 5), (32, 1024, 8), (16, 512, 12)], ids=lambda n: "x".join(map(str, n)))
 def test_separate_y_passes_bitwise(n, precision, monkeypatch):
     """One resident set of groups, each taking many tiles, against one tile per group, bit for bit."""
