@@ -44,10 +44,6 @@ struct NetAct {
 
 namespace {
 
-// Work-groups the weight gradient of one layer is split into (channel blocks x pixel chunks), at
-// most: each chunk writes a partial of the layer's gradient.
-constexpr int kWgradGroups = 256;
-
 __device__ __forceinline__ uint16_t f2bf(float f) { // round to nearest even (finite inputs)
     const uint32_t u = __float_as_uint(f);
     return static_cast<uint16_t>((u + 0x7FFFu + ((u >> 16) & 1u)) >> 16);
@@ -578,24 +574,6 @@ __global__ void k_unpack_output(const float* __restrict__ m, int64_t N, double* 
 }
 
 unsigned nblk(int64_t n, int b = 256) { return static_cast<unsigned>((n + b - 1) / b); }
-
-// Level size, pixel tiles and chunks of a layer's weight gradient
-struct WgradShape {
-    int h, w, tw, tiles_x, tiles, nchunk;
-};
-WgradShape wgrad_shape(int layer, int B, int H, int W) {
-    constexpr int shift[kNetLayers] = {0, 1, 2, 3, 2, 1, 0, 0};
-    WgradShape g{};
-    g.h = H >> shift[layer];
-    g.w = W >> shift[layer];
-    g.tw = g.w <= 8 ? 8 : 16;
-    const int th = 128 / g.tw;
-    g.tiles_x = (g.w + g.tw - 1) / g.tw;
-    g.tiles = g.tiles_x * ((g.h + th - 1) / th);
-    const int blocks = ((kNetCout[layer] + 31) / 32) * ((kNetCin[layer] + 31) / 32);
-    g.nchunk = std::max(1, std::min(B * g.tiles, kWgradGroups / blocks));
-    return g;
-}
 
 } // namespace
 

@@ -4,13 +4,10 @@
 #include <vector>
 
 #include "mafx_internal.hpp"
+#include "net_shapes.hpp"
 
 namespace mafx {
 
-// (in, out) channels of the eight 3x3 convolutions in execution order
-constexpr int kNetLayers = 8;
-constexpr int kNetCin[kNetLayers] = {8, 32, 64, 128, 256, 128, 64, 32};
-constexpr int kNetCout[kNetLayers] = {32, 64, 128, 128, 64, 32, 32, 3};
 constexpr int kNetInputs = 8; // m0 (3) + Ms, A, D, Ku, Bz planes
 
 struct NetAct; // activations of one (B, H, W) shape
