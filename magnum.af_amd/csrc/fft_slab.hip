@@ -418,21 +418,31 @@ template <class C, int NZ, int LOGN> SlabPlan<C> slab_plan_of() {
     using SH = SlabShape<C, NZ, LOGN, LOGS>;
     return {k_slab<C, NZ, LOGN, LOGS, KEEP>, SH::S, SH::Q, SH::BS, SH::LDS};
 }
-// Films of 2, 3, 4 or 8 layers of a power of two of rows.  Left out, where the separate passes are
-// faster: 8 layers of 1024 rows (of 256 or more in FP64), whose sums do not fit the registers, and long
-// columns that leave CUs idle.  Demag field evaluation, us, separate passes -> column pass:
-//   FP32 512 x 64 x 4 44 -> 26, 1024 x 256 x 2 67 -> 49, 512 x 512 x 4 100 -> 90, 1024 x 1024 x 4 353 -> 302;
-//   FP64 512 x 128 x 2 55 -> 36, 512 x 512 x 4 249 -> 218, 1024 x 1024 x 4 1050 -> 883.
-// Left out: FP32 1024 x 1024 x 8 742 -> 915, 100 x 512 x 8 71 -> 77, FP64 512 x 512 x 8 500 -> 632,
-// 100 x 1024 x 4 132 -> 159, 64 x 512 x 3 50 -> 51; and, where a group has a CU to itself, meshes whose
-// last round of columns is nearly empty (260 x 1024 x 2 FP32 76 -> 90, 260 x 256 x 3 FP64 73 -> 83).
+// Films of 2, 3, 4 or 8 layers of a power of two of rows, 64 to 1024; 5, 6 and 7 layers have no kernel here
+// and were not measured.  A group has a CU to itself where its LDS or registers fill one (`heavy`), so the
+// pass takes as long as its rounds of columns, while the separate passes follow the bytes.  It is left out
+// where they were faster, demag field evaluations in us, separate passes against column pass on 256 CUs:
+// - no kernel: the sums do not fit the registers.  FP32 1024 x 1024 x 8 742, 915; FP64 512 x 512 x 8 500, 632;
+// - long columns that leave CUs idle.  FP32 100 x 512 x 8 71, 77; FP64 100 x 1024 x 4 132, 159, 64 x 512 x 3
+//   50, 51;
+// - heavy columns whose last round is nearly empty.  FP32 260 x 1024 x 2 76, 90; FP64 260 x 256 x 3 73, 83;
+// - the two shapes that gain least: FP32 1024 x 2 layers unless nine tenths of the rounds are filled
+//   (600 columns 139, 148; 800 179, 195; 1000 is 2 % faster), and FP64 256 x 3 layers from 3 to 8 rounds
+//   (800 200, 212; 1024 190, 194; 500 is 20 %, 2048 4 % faster).
+// Elsewhere, over 64 to 2048 columns, it is 2 % slower to 83 % faster: FP32 512 x 64 x 4 44, 26; 1024 x 256 x 2
+// 67, 49; 512 x 512 x 4 100, 90; 1024 x 1024 x 4 353, 302; FP64 512 x 128 x 2 55, 36; 512 x 512 x 4 249, 218;
+// 1024 x 1024 x 4 1050, 883.
 template <class C> SlabPlan<C> slab_plan(int nx, int ny, int nz, int cus) {
     constexpr bool F64 = sizeof(C) == sizeof(double2);
     const int hx = nx + 1, rounds = (hx + cus - 1) / cus;
     const bool heavy = ny == 1024 || (ny == 512 && nz == 8) || (F64 && ny == 256 && nz > 2);
     if (nx < cus && (ny == 1024 ? F64 || nz == 4 || 3 * nx < cus : ny == 512 && (nz == 8 || (F64 && nz > 2 && 3 * nx < cus))))
         return {};
-    if (heavy && rounds > 1 && hx % cus > kSlabShared && 4 * hx < 3 * rounds * cus) return {};
+    // a last round of up to kSlabShared columns is spread over the other rounds (slab_rows)
+    const bool partly = rounds > 1 && hx % cus > kSlabShared;
+    if (heavy && partly && 4 * hx < 3 * rounds * cus) return {};
+    if (!F64 && ny == 1024 && nz == 2 && partly && 10 * hx < 9 * rounds * cus) return {};
+    if (F64 && ny == 256 && nz == 3 && hx > 3 * cus && hx < 8 * cus) return {};
     switch (100 * ny + nz) {
 #define MAFX_SLAB(NZ, LOGN) \
     case 100 * (1 << LOGN) + NZ: return slab_plan_of<C, NZ, LOGN>();

@@ -50,7 +50,7 @@ def check(n, precision):
 def test_every_column_kernel(ny, nz, precision, monkeypatch):
     if (ny, nz) in (NO_F64 if precision == "f64" else NO_F32):
         pytest.skip("no column kernel at this size")
-    n = (3 if ny * nz < 2048 else 2, ny, nz)
+    n = (2, ny, nz)
     print(f"\n[column pass] mesh={n} {precision}", flush=True)
     monkeypatch.setenv("MAFX_NUM_CUS", "1")
     rows = check(n, precision)
@@ -86,6 +86,17 @@ def test_shared_columns_on_a_side_stream(precision, monkeypatch):
         h = ctx.heff(state.m_dev)
         side.synchronize()
         assert np.array_equal(h.cpu().numpy().view(np.uint64), ref.view(np.uint64))
+
+
+@pytest.mark.parametrize("n,precision,column", [((27, 1024, 2), "f32", False), ((30, 1024, 2), "f32", True),
+                                                ((25, 256, 3), "f64", False), ((22, 256, 3), "f64", True),
+                                                ((64, 256, 3), "f64", True), ((25, 256, 3), "f32", True)], ids=str)
+def test_rounds_of_columns(n, precision, column, monkeypatch):
+    """With eight CUs: the two shapes that gain least leave the pass to well filled, or few, rounds."""
+    print(f"\n[rounds] mesh={n} {precision}", flush=True)
+    monkeypatch.setenv("MAFX_NUM_CUS", "8")
+    rows = check(n, precision)
+    assert (f"slab_{precision}" in rows) == column, sorted(rows)
 
 
 @pytest.mark.parametrize("precision", ["f64", "f32"])
