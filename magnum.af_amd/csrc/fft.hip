@@ -4,11 +4,12 @@
 //
 // Spectrum layout: planes [comp][kz] of n1 hxs complex values, kx in [0, hx), hx = n0/2 + 1 (R2C
 // half spectrum along x), hxs >= hx padded to 16 columns; ky in [0, n1); kz in [0, nzs) where
-// nzs = nz when the z transform is fused into the tensor product (2 <= nz <= 8) and nzs = n2
-// otherwise.  Inside a plane the columns are grouped in tiles of 4 (tcol, fft_device.hpp):
-// (ky, kx) sits at tcol(kx, 4 n1) + 4 ky.  The tensor spectra use the same planes.  Only rows that can hold non-zero data are touched: the forward x pass
-// writes rows y < ny, z < nz; the forward y pass reads y < ny and writes every ky for z < nz; the
-// fused z kernel reads and writes z < nz; the inverse passes stop at the cropped extent.
+// nzs = nz when the z transform is fused into the tensor product (2 <= nz <= 8) or runs through LDS
+// columns (more layers, z_column_fits) and nzs = n2 otherwise.  Inside a plane the columns are grouped
+// in tiles of 4 (tcol, fft_device.hpp): (ky, kx) sits at tcol(kx, 4 n1) + 4 ky.  The tensor spectra use
+// the same planes.  Only rows that can hold non-zero data are touched: the forward x pass writes rows
+// y < ny, z < nz; the forward y pass reads y < ny and writes every ky for z < nz; the fused z kernel
+// reads and writes z < nz; the inverse passes stop at the cropped extent.
 //
 // Both x passes run a complex FFT of half the padded length on the packed sequence
 // z[n] = x[2n] + i x[2n+1] (the standard real-FFT packing); the zero-padded y passes split the
@@ -1128,9 +1129,8 @@ int lines_per_block(int L, int elems) {
     return W;
 }
 
-const char* nm(const char* f32, const char* f64, size_t csz) { return csz == 8 ? f32 : f64; }
+} // namespace
 
-// Raises a kernel's dynamic LDS limit above the 64 KiB default once per kernel (gfx950: 160 KiB).
 void allow_lds(const void* fn, size_t bytes) {
     static std::mutex mu;
     static std::map<const void*, size_t> granted;
@@ -1142,8 +1142,6 @@ void allow_lds(const void* fn, size_t bytes) {
     MAFX_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
     g = bytes;
 }
-
-} // namespace
 
 // Power-of-two rows below the compile-time shapes: the in-place kernels where their tiles of up to 64 rows
 // give half of the CUs a group, else the per-mesh tiles of fft_mixed.hip (the same sums).  FP64, us, per-mesh

@@ -17,6 +17,12 @@ template <class C> inline const C* tw_of(const FftPlan& p) {
         return reinterpret_cast<const C*>(p.tw32.p);
 }
 
+// Raises a kernel's dynamic LDS limit above the 64 KiB default once per kernel (gfx950: 160 KiB).
+void allow_lds(const void* fn, size_t bytes);
+
+// the profile name of a pass on complex values of csz bytes
+inline const char* nm(const char* f32, const char* f64, size_t csz) { return csz == 8 ? f32 : f64; }
+
 // complex elements of a 64 KiB LDS budget
 template <class C> constexpr int lds_elems() { return 65536 / static_cast<int>(sizeof(C)); }
 

@@ -90,20 +90,6 @@ template <class C> size_t mix_lds(int L, int lines, bool second = true) { return
 // Groups a launch should have before its tiles may grow: three per CU
 int64_t mix_fill(const mafx_ctx* ctx) { return 3 * static_cast<int64_t>(ctx->num_cus); }
 
-void allow_lds(const void* fn, size_t bytes) {
-    static std::mutex mu;
-    static std::map<const void*, size_t> granted;
-    if (bytes <= 65536) return;
-    require(bytes <= kLdsMax, "kernel LDS request exceeds 160 KiB");
-    std::lock_guard<std::mutex> lk(mu);
-    size_t& g = granted[fn];
-    if (g >= bytes) return;
-    MAFX_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(bytes)));
-    g = bytes;
-}
-
-const char* nm(const char* f32, const char* f64, size_t csz) { return csz == 8 ? f32 : f64; }
-
 template <class C>
 __device__ __forceinline__ void stage_twiddles(int M, const C* __restrict__ twh, const C* __restrict__ twL, C* tws, C* twl) {
     for (int t = threadIdx.x; t <= M; t += blockDim.x) {
@@ -166,7 +152,7 @@ template <class C, class T>
 __global__ void __launch_bounds__(512)
     k_mix_x_inv(const C* __restrict__ spec, int64_t hxs, int64_t n1, int64_t n2s, FastDiv Yr, FastDiv Zr, int rows,
                 FastDiv Wd, MixDesc d, FastDiv Mhd, const C* __restrict__ twh, const C* __restrict__ twL,
-                T* __restrict__ out, int Xo, int64_t No, double hscale) {
+                T* __restrict__ out, int Xo, double hscale) {
     extern __shared__ unsigned char smem_raw[];
     const int M = d.L, W = static_cast<int>(Wd.d), row0 = static_cast<int>(blockIdx.x) * W;
     C *A = reinterpret_cast<C*>(smem_raw), *B = A + lds_padded(M * W), *tws = B + lds_padded(M * W);
@@ -555,7 +541,7 @@ template <class C, class T> bool mix_x_inverse(mafx_ctx* ctx, const C* spec, int
                        ctx->stream, spec, ctx->hxs, ctx->n1, n2s, make_fastdiv(static_cast<uint32_t>(g.ny)),
                        make_fastdiv(static_cast<uint32_t>(g.nz)), static_cast<int>(rows), make_fastdiv(W), d,
                        make_fastdiv(static_cast<uint32_t>((g.nx + 1) / 2)), tw_of<C>(ctx->pxh), tw_of<C>(ctx->px), out,
-                       static_cast<int>(g.nx), ctx->N, hscale);
+                       static_cast<int>(g.nx), hscale);
     MAFX_HIP(hipGetLastError());
     return true;
 }

@@ -15,8 +15,8 @@
 // outputs of a class sit at n = j + (Q / 8) q of lane j, the same for every class: the column stays in
 // registers (KEEP) or is read again per class from the caches, and the output sums stay in registers.
 //
-// FP32: the tensor rows of a pair of mirror classes are loaded while the first is transformed, staged in
-// LDS and serve both, so that the tensor is read once and no k-point waits for it.  FP64 (the complex
+// FP32: the tensor rows of a pair of mirror classes, r and S - r, are the same; each class loads them while it
+// is transformed (the second from the caches) and stages them in LDS, so that no k-point waits for them.  FP64 (the complex
 // tensor, 1.6 GB at 1024 x 1024 x 4) and 8 layers: the z transform of a k-point runs on two neighbouring
 // lanes, one for the even and one for the odd kz, which halves the registers it needs; their inverses are
 // added across the pair.
@@ -188,22 +188,20 @@ __global__ void __launch_bounds__((SlabShape<C, NZ, LOGN, LOGS>::BS))
 #pragma unroll
         for (int q = 0; q < 8; ++q) acc[p][q] = C{0, 0};
     __syncthreads(); // the twiddles
-    // mirror classes r and S - r, which share the tensor's rows, one after the other
+    // mirror classes r and S - r, whose tensor rows are the same, one after the other
 #pragma unroll 1
     for (int s = mine; s < s_end; ++s) {
         const int r = s < 2 ? s * (S / 2) : (s & 1) ? S - s / 2 : s / 2;
         const int j = opaque_int(j0); // the stages' addresses are formed per class, not held across it
         f32x4 tv[F64 ? 1 : SH::TV];
         if constexpr (!F64) {
-            // the pair's tensor rows, on their way while its first class is transformed
-            {
-                const f32x4* src = reinterpret_cast<const f32x4*>(
-                    static_cast<const float*>(tens) + (static_cast<int64_t>(kx) * P + s / 2) * SH::TENS);
+            // the pair's tensor rows, on their way while the class is transformed
+            const f32x4* src = reinterpret_cast<const f32x4*>(
+                static_cast<const float*>(tens) + (static_cast<int64_t>(kx) * P + s / 2) * SH::TENS);
 #pragma unroll
-                for (int i = 0; i < SH::TV; ++i) {
-                    const int e = tid + i * SH::BS;
-                    tv[i] = src[e < SH::TENS / 4 ? e : 0];
-                }
+            for (int i = 0; i < SH::TV; ++i) {
+                const int e = tid + i * SH::BS;
+                tv[i] = src[e < SH::TENS / 4 ? e : 0];
             }
         }
         C ws[P]; // w_S^(r p)
@@ -225,12 +223,10 @@ __global__ void __launch_bounds__((SlabShape<C, NZ, LOGN, LOGS>::BS))
 #pragma unroll
         for (int q = 0; q < 8; ++q) rd[(LPL + LPL / 8) * q] = v[q];
         if constexpr (!F64) {
-            {
 #pragma unroll
-                for (int i = 0; i < SH::TV; ++i) {
-                    const int e = tid + i * SH::BS;
-                    if (e < SH::TENS / 4) reinterpret_cast<f32x4*>(ts)[e] = tv[i];
-                }
+            for (int i = 0; i < SH::TV; ++i) {
+                const int e = tid + i * SH::BS;
+                if (e < SH::TENS / 4) reinterpret_cast<f32x4*>(ts)[e] = tv[i];
             }
         }
         __syncthreads();

@@ -458,23 +458,6 @@ void mean_m_noalloc(const double* m, int64_t N, double* out_dev, hipStream_t str
     MAFX_HIP(hipGetLastError());
 }
 
-namespace {
-__global__ void k_axpy_dev(double* __restrict__ y, const double* __restrict__ a, const double* __restrict__ x, int64_t n) {
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * kB + threadIdx.x;
-    if (i < n) y[i] = y[i] + (*a) * x[i];
-}
-} // namespace
-
-void dot_dev(mafx_ctx* ctx, const double* a, const double* b, int64_t n, double* out_dev) {
-    lbfgs_flush(ctx);
-    const unsigned nb = red_blocks(n);
-    ProfScope ps(ctx, "dot_f64", 16.0 * n);
-    hipLaunchKernelGGL(k_dot, dim3(nb), dim3(kB), 0, ctx->stream, a, b, n, ctx->partials.as<double>());
-    hipLaunchKernelGGL(k_final, dim3(1), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(), static_cast<int>(nb),
-                       1, 1, out_dev);
-    MAFX_HIP(hipGetLastError());
-}
-
 void reduce_slots(mafx_ctx* ctx, int64_t nblocks, int nslots, int nsum, const double* a, const double* b, int64_t n) {
     lbfgs_flush(ctx);
     const unsigned nb = red_blocks(n);
@@ -488,21 +471,12 @@ void reduce_slots(mafx_ctx* ctx, int64_t nblocks, int nslots, int nsum, const do
                        nblocks, nslots, nsum, part2, static_cast<int>(nb), ctx->host_scal);
     MAFX_HIP(hipGetLastError());
 }
-void max_abs_dev(mafx_ctx* ctx, const double* a, int64_t n, double* out_dev) {
-    lbfgs_flush(ctx);
-    const unsigned nb = red_blocks(n);
-    ProfScope ps(ctx, "maxabs_f64", 8.0 * n);
-    hipLaunchKernelGGL(k_maxabs, dim3(nb), dim3(kB), 0, ctx->stream, a, n, ctx->partials.as<double>());
-    hipLaunchKernelGGL(k_final, dim3(1), dim3(kB), 0, ctx->stream, ctx->partials.as<double>(), static_cast<int>(nb),
-                       1, 0, out_dev);
-    MAFX_HIP(hipGetLastError());
-}
 
 namespace {
 // One step of the LBFGS two-loop recursion with the next step's dot product: qi = q_in + (*coef) v
 // (no axpy when coef is null), then qi = scale qi when do_scale, stored as q_out = qi or, negate,
 // q_out = -qi; and partials of dnext . qi.  Every expression and the element-to-thread mapping are
-// those of k_axpy_dev, k_scale and k_dot, so the results equal the unfused sequence bit for bit.
+// those of an axpy pass, k_scale and k_dot, so the results equal the unfused sequence bit for bit.
 // PMODE >= 1: the coefficient is the previous step's, formed here from its partials ppart[0..pnb)
 // with k_final_coef<PMODE>'s tree and expressions (every work-group forms the same value; group 0
 // also stores the dot product, alpha_i and the coefficient as k_final_coef would).  PMODE = -1:
@@ -699,11 +673,6 @@ void lbfgs_pair(mafx_ctx* ctx, const double* m, const double* x_old, const doubl
 
 void neg_copy(mafx_ctx* ctx, double* y, const double* x, int64_t n) {
     hipLaunchKernelGGL(k_neg, dim3(grid_for(n, kB)), dim3(kB), 0, ctx->stream, y, x, n);
-    MAFX_HIP(hipGetLastError());
-}
-
-void axpy_dev(mafx_ctx* ctx, double* y, const double* a_dev, const double* x, int64_t n) {
-    hipLaunchKernelGGL(k_axpy_dev, dim3(grid_for(n, kB)), dim3(kB), 0, ctx->stream, y, a_dev, x, n);
     MAFX_HIP(hipGetLastError());
 }
 

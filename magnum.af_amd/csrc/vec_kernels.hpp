@@ -19,14 +19,9 @@ void sub(mafx_ctx* ctx, double* out, const double* a, const double* b, int64_t n
 void copy(mafx_ctx* ctx, double* dst, const double* src, int64_t n);
 int64_t reduction_partials_needed(int64_t n);
 int64_t reduction_partials_extra(); // doubles at the end of the partials, beside an evaluation's own
-// Device-side scalars (no host synchronisation): *out_dev = a . b and max |a| with the kernels and
-// reduction tree of dot() / max_abs(), y += (*a_dev) x.
-void dot_dev(mafx_ctx* ctx, const double* a, const double* b, int64_t n, double* out_dev);
-void max_abs_dev(mafx_ctx* ctx, const double* a, int64_t n, double* out_dev);
 // The evaluation's slots [0, nslots) to ctx->host_scal (sums for s < nsum, then maxima) and, with a,
-// a . b and max |a| to the two slots behind them, each bit for bit as dot_dev / max_abs_dev form it.
+// a . b and max |a| to the two slots behind them, each bit for bit as dot() / max_abs() form it.
 void reduce_slots(mafx_ctx* ctx, int64_t nblocks, int nslots, int nsum, const double* a, const double* b, int64_t n);
-void axpy_dev(mafx_ctx* ctx, double* y, const double* a_dev, const double* x, int64_t n);
 // LBFGS fused vector work, bit for bit the unfused sequence's results:
 // lbfgs_fused: q_out = (q_in + (*coef_dev) v) [* scale] (negated when `negate`), *out_dev = dnext . q
 //   (before negation), with dot()'s tree; coef_dev null skips the axpy.  q_out may alias q_in.
