@@ -154,9 +154,10 @@ struct mafx_ctx {
     int precision{MAFX_F64};
     int num_cus{256};         // compute units of the current device (persistent grids)
     // RK stage inputs are formed in the per-cell pass from this many cells on where that pass walks z
-    // columns of several layers (below it has too few lanes to hide the extra loads: 512 x 32 x 4 297
-    // against 318 us a step), and always where it has a lane per cell (1024 x 256 x 1 350 -> 329,
-    // 100 x 25 x 1 210 -> 203); MAFX_RK_FUSE_MIN_CELLS overrides it
+    // columns of several layers (below it has too few lanes to hide the extra loads: an FP64 DP45 step at
+    // 1024 x 128 x 4 880 against 908 us, 512 x 256 x 4 1056 against 1072; with two layers the two forms are
+    // within 2 %), and always where it has a lane per cell (1024 x 256 x 1 350 -> 329, 100 x 25 x 1 210 ->
+    // 203); MAFX_RK_FUSE_MIN_CELLS overrides it
     int64_t rk_fuse_min_cells{int64_t{1} << 20};
     // MAFX_F32_FIELD integrators keep their stage derivatives k_j in FP32 (MAFX_RK_K64=1: FP64)
     bool rk_k32{true};
