@@ -14,9 +14,9 @@ from test_gpu_parity import build, mf, normwise, rand_m
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [(ny, nz) for ny in (64, 128, 256, 512, 1024) for nz in (2, 3, 4, 8)]
-NO_F32 = {(1024, 8)}
-NO_F64 = {(256, 8), (512, 8), (1024, 8)}
+# every (rows, layers) with a kernel: FP32 without 1024 x 8, FP64 without 8 layers of 256 rows or more
+KERNELS = [(ny, nz, p) for p in ("f32", "f64") for ny in (64, 128, 256, 512, 1024) for nz in (2, 3, 4, 8)
+           if nz < 8 or ny < (1024 if p == "f32" else 256)]
 
 
 def field_twice(state, term, precision):
@@ -45,11 +45,8 @@ def check(n, precision):
     return rows
 
 
-@pytest.mark.parametrize("precision", ["f64", "f32"])
-@pytest.mark.parametrize("ny,nz", SHAPES)
+@pytest.mark.parametrize("ny,nz,precision", KERNELS)
 def test_every_column_kernel(ny, nz, precision, monkeypatch):
-    if (ny, nz) in (NO_F64 if precision == "f64" else NO_F32):
-        pytest.skip("no column kernel at this size")
     n = (2, ny, nz)
     print(f"\n[column pass] mesh={n} {precision}", flush=True)
     monkeypatch.setenv("MAFX_NUM_CUS", "1")
