@@ -152,8 +152,11 @@ int mafx_device_count(int* count);
  * precision.  Uploads parameters, builds the demag / dipole tensor on the GPU in FP64
  * (demag_field.cpp:104-147), plans the FFTs and allocates the workspace.  Replaces the
  * construction of the reference's terms plus State::Ms/Ms_field.  Reads MAFX_NUM_CUS (CU count
- * for the persistent transform grids; default: the device's) and, with MAFX_TERM_CACHING,
- * MAFX_CACHE_DIR / MAFX_CACHE_MAX_BYTES. */
+ * that sizes the persistent transform grids and chooses between kernels by how far they fill the chip;
+ * default: the device's) and, with MAFX_TERM_CACHING, MAFX_CACHE_DIR / MAFX_CACHE_MAX_BYTES.  Set-up
+ * holds more device memory than the finished context: the real-space tensor while the spectrum is built,
+ * and, for films of a few layers, a second copy of the tensor (also of one read from the cache) while it
+ * is stored anew in the order their column pass reads. */
 int mafx_ctx_create(const mafx_mesh* mesh, double Ms, const double* Ms_field_host,
                     const mafx_term_desc* terms, int nterms, int precision, mafx_ctx** out);
 int mafx_ctx_destroy(mafx_ctx* ctx);

@@ -262,8 +262,8 @@ int mafx_ctx_create(const mafx_mesh* mesh, double Ms, const double* Ms_field_hos
         if (cus > 0) ctx->num_cus = cus;
         // MAFX_RK_K64=1 keeps the FP32-field integrator's stage derivatives in FP64
         if (const char* e = std::getenv("MAFX_RK_K64")) ctx->rk_k32 = std::atoi(e) == 0;
-        // MAFX_NUM_CUS overrides the CU count that sizes the persistent grids (tuning, and tests
-        // that make each resident group take many tiles on small meshes)
+        // MAFX_NUM_CUS overrides the CU count that sizes the persistent grids and chooses between kernels
+        // (tuning, and tests that reach them on small meshes)
         if (const char* e = std::getenv("MAFX_NUM_CUS")) {
             const int v = std::atoi(e);
             if (v > 0) ctx->num_cus = v;
